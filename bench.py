@@ -343,14 +343,12 @@ def main() -> int:
     if not args.no_split:
         split = harness_split(forward, backward, reset, min(args.steps, 20))
 
-    # Roofline of the blend backward: one hds_render_backward call runs its two kernels (back-to-front
-    # geometry/colour gradients, front-to-back feature gradients) side by side on two streams. The
-    # duration is the pair's span, first start to last end, from the HIP events the library records
-    # on each kernel's own stream over the timed region (rocprofv3's kernel trace gives the same
-    # span); the per-kernel means, each longer than when run alone, are reported beside it.
+    # Roofline of the blend backward: one hds_render_backward_rows call lists each block's gaussians,
+    # replays the blocks back to front and sums the gradient rows. The duration is from the first kernel's
+    # start to the last one's end.
     bwd_names, bwd_ms = backward_span(kernels, kprof.timeline)
     achieved = alg["render_backward"] / (bwd_ms * 1e-3) / 1e9
-    roofline = {"kernel": " + ".join(bwd_names) + (" (side by side, one hds_render_backward call)"
+    roofline = {"kernel": " + ".join(bwd_names) + (" (one hds_render_backward_rows call)"
                                                    if len(bwd_names) > 1 else ""),
                 "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
@@ -422,17 +420,14 @@ def main() -> int:
 
 
 # The blend backward's kernels: the only launches the library times inside the timed region.
-BACKWARD_KERNELS = ("backward_geometry_kernel", "backward_features_kernel")
+BACKWARD_KERNELS = ("backward_lists_kernel", "backward_geometry_kernel", "backward_features_kernel")
 
 
 def backward_span(kernels: dict, timeline) -> tuple[list[str], float]:
     """The blend backward's kernels in the timed region and the mean duration of one
-    hds_render_backward call: with two kernels side by side on two streams, their span (first start
-    to last end); with one, its mean."""
+    hds_render_backward_rows call: from the start of its first kernel to the end of its last."""
     names = [k for k in BACKWARD_KERNELS if k in kernels]
-    if len(names) == 2:
-        return names, concurrent_span_ms(timeline, *names)
-    return names, kernels[names[0]]["mean_ms"]
+    return names, call_span_ms(timeline, names)
 
 
 def harness_split(fn_fwd, fn_bwd, reset, samples: int) -> dict:
@@ -700,15 +695,11 @@ def config_cpu_baseline(wl, frame, index: int, ranges, samples: int) -> dict:
     return record
 
 
-def concurrent_span_ms(timeline, first: str, second: str) -> float:
-    """Mean over calls of (later end - earlier start) of two kernels launched together: each `first`
-    launch is paired with the `second` launch that starts nearest to it."""
-    a = [(t0, t1) for name, t0, t1 in timeline if name == first]
-    b = [(t0, t1) for name, t0, t1 in timeline if name == second]
-    spans = []
-    for s0, e0 in a:
-        s1, e1 = min(b, key=lambda se: abs(se[0] - s0))
-        spans.append(max(e0, e1) - min(s0, s1))
+def call_span_ms(timeline, names: list[str]) -> float:
+    """Mean over calls of (last end - first start) of kernels that every call launches once each, on one
+    stream: the i-th launches of all `names` belong to the i-th call."""
+    launches = [[(t0, t1) for name, t0, t1 in timeline if name == n] for n in names]
+    spans = [max(e for _, e in call) - min(s for s, _ in call) for call in zip(*launches)]
     return sum(spans) / len(spans)
 
 

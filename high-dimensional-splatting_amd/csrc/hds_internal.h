@@ -274,6 +274,15 @@ __device__ static inline int hds_xcd_tile(int block, int tiles_x, int num_tiles)
 	return tx < tiles_x && ty < tiles_y ? ty * tiles_x + tx : -1;
 }
 
+/* The same order for work-groups of one 8x8 block each: the four blocks of a tile are consecutive on the
+ * tile's XCD. Returns 4 * tile + block (block = x half + 2 * y half), or -1 for padding. */
+static inline unsigned hds_xcd_block_grid(int tiles_x, int num_tiles) { return 4 * hds_xcd_grid(tiles_x, num_tiles); }
+__device__ static inline int hds_xcd_block(int block, int tiles_x, int num_tiles) {
+	const int xcd = block % HDS_XCDS, r = block / HDS_XCDS;
+	const int tile = hds_xcd_tile((r >> 2) * HDS_XCDS + xcd, tiles_x, num_tiles);
+	return tile < 0 ? -1 : 4 * tile + (r & 3);
+}
+
 /* acc += A * B with A, B given as split-bf16 pairs (small terms first). */
 __device__ static inline hds_f32x4 hds_mfma_split(const hds_bf16x8& a_hi, const hds_bf16x8& a_lo,
 												  const hds_bf16x8& b_hi, const hds_bf16x8& b_lo,

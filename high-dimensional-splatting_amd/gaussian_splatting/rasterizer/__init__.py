@@ -3,10 +3,9 @@
 Mirrors gaussian_splatting/rasterizer/__init__.py of the reference: the same `rasterize` signature and
 return values, the `RasterizeGaussians` autograd node, the `FEATURE_SLICE_WIDTH` knob and
 `_get_rasterizer()`, which here returns the ctypes binding of the HIP library instead of a JIT-built
-CUDA extension. The forward renders RGB and features in one tile walk. The backward runs two tile
-kernels side by side: a back-to-front replay for the geometry gradients (means2D, conics, opacities,
-colours), and a front-to-back replay that contracts the blend weights with dL/dF for the feature
-gradients.
+CUDA extension. The forward renders RGB and features in one tile walk. The backward replays each 8x8 pixel
+block back to front for all gradients at once (means2D, conics, opacities, colours, features), stores them
+as one row per (gaussian, block) and sums every gaussian's rows.
 """
 from __future__ import annotations
 
@@ -86,7 +85,7 @@ class RasterizeGaussians(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_image, grad_features=None):
-        """Gradients of the blend for RGB and features from one library call (two kernels side by side).
+        """Gradients of the blend for RGB and features from one library call.
 
         Returns:
             Gradients for means2D, conics, colors, opacities and features; None for depths, radii,

@@ -61,6 +61,9 @@ PROTOTYPES = {
                                    _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_render_backward_accumulate": (_i32, [_i64, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp,
                                               _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "hds_render_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
+    "hds_render_backward_rows": (_i32, [_i64, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp,
+                                        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _vp, _sz, _vp]),
     "hds_ssim_forward": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_ssim_backward": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_densification_stats": (_i32, [_i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
@@ -259,6 +262,9 @@ class HipRasterizer:
     # of it the last frame's longest list may reach for bin_async to choose that binning.
     TILE_ORDER_MAX = 4096
     TILE_ORDER_MARGIN = 0.9
+
+    # Most bytes of gradient rows that the blend backward stores; it adds the gradients of the rest atomically.
+    ROWS_MAX_BYTES = 8 << 30
 
     def __init__(self) -> None:
         self.lib = load_library()
@@ -567,10 +573,9 @@ class HipRasterizer:
     def render_backward(self, means2D, conic4, color_opacity4, values_sorted, tile_ranges, final_T, n_contrib,
                         width, height, grad_image=None, background=None, features=None, grad_feature_image=None,
                         slice_width=None, want_feature_grad=True, prezeroed=None):
-        """The blend backward (backward.cu:7-164 + features.cu:350-542): geometry gradients from a
-        back-to-front replay, feature gradients from a front-to-back replay beside it. `prezeroed` is the
-        buffers of gradient_buffers, zeroed by earlier work on the current stream (render(clear=...)):
-        the gradients are then added into those buffers instead of into buffers zeroed here.
+        """The blend backward (backward.cu:7-164 + features.cu:350-542): hds_render_backward_rows where its workspace
+        fits, else the atomic hds_render_backward. `prezeroed` is the buffers of gradient_buffers, zeroed by
+        earlier work on the current stream (render(clear=...)), to write the gradients into.
 
         Returns (grad_means2D [N,2], grad_conics [N,3], grad_colors [N,3] or None, grad_opacities [N,1],
         grad_features [N,C] or None).
@@ -595,24 +600,42 @@ class HipRasterizer:
                 g_feat = None
             elif g_feat.shape != (n, channels):
                 raise RuntimeError(f"prezeroed grad_features {tuple(g_feat.shape)} != ({n}, {channels})")
-            entry = self.lib.hds_render_backward_accumulate
         else:
-            # hds_render_backward zeroes the outputs itself before its atomics add into them.
             f32 = dict(device=dev, dtype=torch.float32)
             g_means = torch.empty((n, 2), **f32)
             g_conics = torch.empty((n, 3), **f32)
             g_colors = torch.empty((n, 3), **f32) if grad_image is not None else None
             g_opac = torch.empty((n, 1), **f32)
             g_feat = torch.empty((n, channels), **f32) if want_feat else None
-            entry = self.lib.hds_render_backward
-        with torch.cuda.device(dev):
-            self._run("render_backward", lambda: entry(
-                n, int(width), int(height), channels, slice_width or 0, _ptr(tile_ranges), _ptr(values_sorted),
+        args = (n, int(width), int(height), channels, slice_width or 0, _ptr(tile_ranges), _ptr(values_sorted),
                 values_sorted.numel(), _ptr(_dev(means2D, "means2D")), _ptr(conic4), _ptr(color_opacity4),
                 _ptr(background), _ptr(final_T), _ptr(n_contrib), _ptr(grad_image), _ptr(features),
-                _ptr(grad_feature_image), _ptr(g_means), _ptr(g_conics), _ptr(g_colors), _ptr(g_opac), _ptr(g_feat),
-                _stream(dev)))
+                _ptr(grad_feature_image), _ptr(g_means), _ptr(g_conics), _ptr(g_colors), _ptr(g_opac), _ptr(g_feat))
+        with torch.cuda.device(dev):
+            rows, workspace = self._backward_workspace(n, int(width), int(height), channels, slice_width or 0, want_feat,
+                                                       values_sorted.numel(), dev)
+            if workspace is not None:
+                self._run("render_backward", lambda: self.lib.hds_render_backward_rows(
+                    *args, int(prezeroed is not None), rows, _ptr(workspace), workspace.numel(), _stream(dev)))
+            else:
+                entry = (self.lib.hds_render_backward if prezeroed is None
+                         else self.lib.hds_render_backward_accumulate)
+                self._run("render_backward", lambda: entry(*args, _stream(dev)))
         return g_means, g_conics, g_colors, g_opac, g_feat
+
+    def _backward_workspace(self, n, width, height, channels, slice_width, want_feat, pairs, dev):
+        """(row capacity, workspace) of hds_render_backward_rows: room for the most gradient rows the pairs can have
+        (four per (tile, gaussian) pair, one per 8x8 block of the tile; 1.4 to 1.9 are in use on scenes of small
+        gaussians, far fewer where most pairs are occluded), or for ROWS_MAX_BYTES of them where that is less; no
+        workspace when the memory is not there."""
+        row_bytes = 4 * (channels if want_feat else 0) + 64 * (channels // slice_width if channels else 1)
+        rows = min(4 * pairs, self.ROWS_MAX_BYTES // row_bytes, 2**30 - 1024)
+        size = int(self.lib.hds_render_backward_workspace_bytes(n, width, height, channels, slice_width, int(want_feat),
+                                                                pairs, rows))
+        try:
+            return rows, torch.empty(size, device=dev, dtype=torch.uint8)
+        except torch.cuda.OutOfMemoryError:
+            return 0, None
 
     # -- the reference extension's rasterize* entry points --------------------------------------
 

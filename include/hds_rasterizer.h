@@ -266,6 +266,23 @@ HDS_API int hds_render_backward_accumulate(
 	const float* grad_image, const float* features, const float* grad_feature_image, float* grad_means2D,
 	float* grad_conics, float* grad_colors, float* grad_opacities, float* grad_features, hds_stream_t stream);
 
+/* Workspace of hds_render_backward_rows (want_features: grad_features is given; channels 0: no features). */
+HDS_API size_t hds_render_backward_workspace_bytes(int64_t n, int width, int height, int channels, int slice_width,
+												   int want_features, int64_t num_pairs, int64_t row_capacity);
+
+/* hds_render_backward through a workspace: the blend's gradients of each (gaussian, 8x8 pixel block) are stored as
+ * a row, and each gaussian's rows are summed by a second pass, instead of being added atomically. At most
+ * row_capacity rows (up to 2^30 - 1024) are stored; the gradients of rows past that are added atomically. zeroed != 0: the
+ * gradient outputs hold zeros already. The workspace (16-byte aligned, its contents do not matter) is free
+ * again when the stream has run the call. */
+HDS_API int hds_render_backward_rows(
+	int64_t n, int width, int height, int channels, int slice_width, const int32_t* tile_ranges,
+	const int32_t* values_sorted, int64_t num_pairs, const float* means2D, const float* conic4,
+	const float* color_opacity4, const float* background, const float* final_T, const int32_t* n_contrib,
+	const float* grad_image, const float* features, const float* grad_feature_image, float* grad_means2D,
+	float* grad_conics, float* grad_colors, float* grad_opacities, float* grad_features, int zeroed,
+	int64_t row_capacity, void* workspace, size_t workspace_bytes, hds_stream_t stream);
+
 /* Zeroes `count` floats at p (16-byte aligned, count a multiple of 4) on `stream` with at most
  * `max_workgroups` work-groups of 256 threads (0: as many as fill the device), so that a large fill
  * enqueued beside latency-bound kernels takes only part of the CUs. The zero-initialised buffers of
