@@ -195,6 +195,7 @@ __device__ static inline float hds_wave_reduce_scatter8(float v[8], int lane) {
 /* ------------------------------------------------------------------------------------------- */
 
 typedef __bf16 hds_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float hds_f32x2 __attribute__((ext_vector_type(2)));
 typedef float hds_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t hds_u32x4 __attribute__((ext_vector_type(4)));
 

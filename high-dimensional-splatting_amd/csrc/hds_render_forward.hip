@@ -1,26 +1,31 @@
-// Front-to-back blend of RGB and C feature channels in one tile walk.
+// Front-to-back blend of RGB and C feature channels in one walk.
 //
-// Work-group = one 16x16 tile (and one slice of S <= 128 channels); wave w owns the 8x8 block
-// ((w & 1) * 8, (w >> 1) * 8) and lane l the pixel (l & 7, l >> 3) of it. Gaussians of the tile's
-// sorted list are staged 64 at a time in LDS (geometry, culling box and the slice's feature rows as
-// raw fp32, split into bf16 operands when read); each wave ballots which of the 64 box-hit its block
-// and walks only those, in order, updating T, RGB and n_contrib per lane exactly as render_gaussians does
-// (forward.cu:181-225): alpha = min(0.99, op * exp(-m/2)), skip below 1/255, stop before T would
-// drop below 1e-4, n_contrib = 1-based list index of the last blended gaussian.
+// Work-group = one wave = one 8x8 block of a tile (and one slice of S <= 128 channels), lane l the pixel (l & 7,
+// l >> 3) of it. The wave tests 64 entries of the tile's sorted list at a time against its block, keeps those that
+// can reach it, in order, and takes them 16 at a time, updating T, RGB and n_contrib per lane exactly as
+// render_gaussians does (forward.cu:181-225): alpha = min(0.99, op * exp(-m/2)), skip below 1/255, stop before T
+// would drop below 1e-4, n_contrib = 1-based list index of the last blended gaussian.
 //
-// Features: the wave's box-hits are taken 16 at a time, in list order, as the K dimension of
+// Features: the 16 hits are, in list order, the K dimension of
 //   out[c][px] += sum_k F[k][c] * W[k][px],
 // one v_mfma_f32_32x32x16_bf16 per 32 channels x 32 pixels, both operands in split-bf16 (3 MFMAs
 // per tile, ~2^-16 relative error; CDNA4 has no TF32). Each lane keeps its own pixel's 16 weights
 // w = alpha * T (0 where it did not blend) in registers as packed bf16 pairs; one
 // v_permlane32_swap per register pair then forms the B operands of the two 32-pixel halves, so the
-// weights never touch LDS. The 16-hit groups depend on geometry only and the batch size is fixed,
-// so each output channel sees the same operation sequence whatever C or the slicing is: channels
-// are bitwise independent and RGB is bitwise equal with or without features (the properties the
-// reference's tests/test_properties.py pins). The accumulators take S registers per lane (ordinary
-// VGPRs: the compiler assigns no AGPRs here); with the walk's registers the 128-channel slice needs
-// about 240 and runs two waves per SIMD, the 64-channel slice three, the 32-channel slice three with
-// RGB (four would cap it at 128 registers, which spills) and four without.
+// weights never touch LDS. The 16-hit groups depend on geometry only, so each output channel sees the same
+// operation sequence whatever C or the slicing is: channels are bitwise independent and RGB is bitwise equal with or
+// without features (the properties the reference's tests/test_properties.py pins). The accumulators take S registers
+// per lane (ordinary VGPRs: the compiler assigns no AGPRs here), so the 128-channel slice runs two waves per
+// SIMD, the 64-channel slice three, the 32-channel slice four.
+//
+// Bound by VALU issue (about 35 operations per hit and 230 per group of 16 for the split operands) and, where the
+// feature image or the cleared range is large, by stores. Against one work-group per tile, whose four waves shared a
+// staged batch and met at a barrier after each: no wave waits for another, groups run on over batches
+// (145k full ones instead of 226k at 1.18M gaussians, 979x546), rows no block can see are not copied, and a wave's
+// slot is free when its block is done. Alphas are evaluated four at a time before the chain through T, which has
+// no branch but one per four hits for pixels that stop there. The image leaves in whole lines, non-temporal.
+// At 979x546: C = 32, 200k gaussians, 0.100 -> 0.070 ms; 1.18M: RGB 0.230 -> 0.187, C = 128 0.62 -> 0.49; at 4M,
+// 1920x1080, C = 256: 1.61 -> 1.37.
 #include <cstdlib>
 
 #include "hds_internal.h"
@@ -29,9 +34,17 @@
 
 namespace {
 
-constexpr int kBatch = 64;  // gaussians staged per LDS batch = one ballot per wave
-constexpr int kGroup = 16;  // K of one MFMA: box-hits per group
+constexpr int kBatch = 64;  // entries of the tile's list tested together, one per lane
+constexpr int kGroup = 16;  // K of one MFMA: hits per group
+constexpr int kHits = kGroup + kBatch;  // most hits pending, and more than a group reads past the last
 constexpr int kIlp = 4;     // hits whose alpha is evaluated together
+constexpr float kDone = 2.0f;  // alpha that none reaches
+
+// Waits for this wave's outstanding vector-memory operations, LDS copies included.
+__device__ inline void wait_vmem() {
+	__builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), which the compiler's own count knows of
+	asm volatile("" ::: "memory");
+}
 
 struct RenderArgs {
 	int width, height, tiles_x, channels, num_tiles;
@@ -50,13 +63,24 @@ struct RenderArgs {
 	int64_t clear4;
 };
 
+// Feature rows of a group in LDS, S floats each, in the order of their copy: wave instruction i brings 1 KB, in its
+// lower half rows i * kRowsPerHalf .. of hits 0-7 and in its upper half the same rows of hits 8-15.
+template <int S>
+struct RowLayout {
+	static constexpr int kLanes = S / 4;                   // lanes (16 bytes each) per row
+	static constexpr int kRowsPerHalf = 32 / kLanes;       // rows per half instruction
+	static constexpr int kOps = (kGroup / 2) / kRowsPerHalf;
+	// Float offset of row 8 h + j.
+	static __device__ constexpr int at(int h, int j) { return (j / kRowsPerHalf) * 256 + h * 128 + (j % kRowsPerHalf) * S; }
+};
+
 // acc[m][cb] += F^T W for one group. w_hi / w_lo hold this lane's pixel's packed weights for
 // positions (2i, 2i+1); after the swaps, words 0-3 are the B operand of pixels 0-31 and words 4-7
 // that of pixels 32-63. A = features: lane = (channel lane % 32, positions 8 (lane / 32) + 0..7),
-// read as raw fp32 from the staged rows (S floats each) and split here.
+// read as raw fp32 from the staged rows and split here.
 template <int S>
 __device__ inline void flush_group(hds_f32x16 (&acc)[2][S / 32], uint32_t (&w_hi)[8], uint32_t (&w_lo)[8],
-								   const int (&slot)[kGroup], const float* feat, int lane) {
+								   const float* feat, int lane) {
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		const auto h = __builtin_amdgcn_permlane32_swap(w_hi[i], w_hi[4 + i], false, false);
@@ -72,213 +96,272 @@ __device__ inline void flush_group(hds_f32x16 (&acc)[2][S / 32], uint32_t (&w_hi
 		b_hi[m] = __builtin_bit_cast(hds_bf16x8, hds_u32x4{w_hi[4 * m], w_hi[4 * m + 1], w_hi[4 * m + 2], w_hi[4 * m + 3]});
 		b_lo[m] = __builtin_bit_cast(hds_bf16x8, hds_u32x4{w_lo[4 * m], w_lo[4 * m + 1], w_lo[4 * m + 2], w_lo[4 * m + 3]});
 	}
-	const bool upper = lane >= 32;
-	const int col = lane & 31;
-	int row[8];
-#pragma unroll
-	for (int j = 0; j < 8; j++) {
-		// Select the values, not the array half: an indexed pointer select would put slot in scratch.
-		const int lo = slot[j], hi = slot[8 + j];
-		row[j] = (upper ? hi : lo) * S + col;
-	}
+	const float* const mine = feat + RowLayout<S>::at(lane >> 5, 0) + (lane & 31);
 #pragma unroll
 	for (int cb = 0; cb < S / 32; cb++) {
 		float v[8];
 #pragma unroll
-		for (int j = 0; j < 8; j++) v[j] = feat[row[j] + 32 * cb];
+		for (int j = 0; j < 8; j++) v[j] = mine[RowLayout<S>::at(0, j) + 32 * cb];
 		hds_bf16x8 a_hi, a_lo;
 		hds_split8(v, a_hi, a_lo);
 #pragma unroll
 		for (int m = 0; m < 2; m++) acc[m][cb] = hds_mfma32_split(a_hi, a_lo, b_hi[m], b_lo[m], acc[m][cb]);
+		asm volatile("" : "+v"(acc[0][cb]), "+v"(acc[1][cb]));  // summed here, not on either side of the loop's exit
 	}
 }
 
-// Per-lane state of the walk.
+// Stages group hits first .. first + rows - 1 of the list: feature rows into feat, colours into rgb. Rows past the
+// last hit (only a walk's last group has any) become zeros.
+template <int S, bool RGB>
+__device__ inline void stage_group(float* feat, float* rgb, const RenderArgs& a, const int* gids, int first, int rows, int c0) {
+	const int lane = (int)hds_opaque(threadIdx.x);  // what follows from it is worked out here, not held through the walk
+	if (rows < kGroup) {
+		// The buffer is idle: zeros first, then what there is.
+		if constexpr (S > 0)
+			for (int i = lane; i < kGroup * S / 4; i += 64) reinterpret_cast<hds_f32x4*>(feat)[i] = hds_f32x4{};
+		if constexpr (RGB)
+			if (lane < 3 * kGroup) rgb[lane] = 0.0f;
+		__builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+		asm volatile("" ::: "memory");
+	}
+	if constexpr (S > 0) {
+		using L = RowLayout<S>;
+		const int row0 = 8 * (lane >> 5) + (lane & 31) / L::kLanes;
+		const float* const src = a.features + c0 + 4 * (lane % L::kLanes);
+#pragma unroll
+		for (int i = 0; i < L::kOps; i++) {
+			const int row = row0 + i * L::kRowsPerHalf;
+			if (row < rows)
+				__builtin_amdgcn_global_load_lds(src + (size_t)gids[first + row] * a.channels, (hds_lds_void*)(feat + 256 * i), 16, 0, 0);
+		}
+	}
+	if constexpr (RGB) {
+		if (lane < rows) {
+			const float4* const color = a.color_op4 + gids[first + lane];
+			__builtin_amdgcn_global_load_lds(&color->x, (hds_lds_void*)(rgb), 4, 0, 0);
+			__builtin_amdgcn_global_load_lds(&color->y, (hds_lds_void*)(rgb + kGroup), 4, 0, 0);
+			__builtin_amdgcn_global_load_lds(&color->z, (hds_lds_void*)(rgb + 2 * kGroup), 4, 0, 0);
+		}
+	}
+}
+
+// Per-lane state of the walk. A gaussian blends where its alpha reaches `reach`: 1/255 until the pixel is done (or
+// from the start outside the image), 2 afterwards.
 struct Pixel {
 	float T;
-	bool done;
-	int last;
+	float reach;
+	int n_contrib;
 	float r, g, b;
 };
 
-// Occupancy: S accumulators per lane plus the walk's registers, two waves per SIMD with features.
-//
-// Pipeline per batch b: the records and feature rows of batch b+1 are copied into the other slot by
-// LDS DMA while b is walked, and the gids of b+2 are read; one barrier, after each wave has waited
-// for its copies, hands the next batch over.
+// hds_render_clear: every work-group zeroes a share of the caller's range before its walk. The walks leave most of the
+// HBM bandwidth unused, so the stores drain beside those of other waves instead of in a fill launch of their own;
+// non-temporal, so that the zeros do not push feature rows out of L2. (After the walk: 1.43 ms instead of 1.37 at 4M
+// gaussians, C = 256; a piece per group: 1.72 instead of 1.65 before the image's stores became whole lines.)
+__device__ inline void clear_share(const RenderArgs& a, int lane) {
+	constexpr int kPiece = 256;  // 4 KB dealt out in turn
+	const int64_t stride = (int64_t)gridDim.x * gridDim.y * kPiece;
+	hds_f32x4* const clear = reinterpret_cast<hds_f32x4*>(a.clear);
+	for (int64_t e = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kPiece + lane; e < a.clear4; e += stride) {
+#pragma unroll
+		for (int k = 0; k < kPiece; k += 64)
+			if (e + k < a.clear4) __builtin_nontemporal_store(hds_f32x4{}, clear + e + k);
+	}
+}
+
+// A wave is a work-group of its own: nothing in it waits for another. Per group of 16 hits it tests batches of entries
+// until so many are pending (a batch's records are read while the one before is worked on), issues the copies
+// of the group's feature rows and colours, evaluates the alphas and the chain through T while those are on their way,
+// and then adds the colours and features.
 template <int S, bool RGB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2 : (S == 64 || RGB) ? 3 : 4))) void render_forward_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2 : S == 64 ? 3 : 4))) void render_forward_kernel(
 	const RenderArgs a) {
 	constexpr int kNcb = S > 0 ? S / 32 : 1;
-	constexpr int kRows = S > 0 ? (kBatch + 1) * S : 1;
 
-	// Gaussian ids of batches b, b+1, b+2 (slot b % 3).
-	__shared__ int s_gid[3][kBatch];
-	// Records and feature rows of the batch being walked and of the next one; feature row kBatch
-	// stays zero (positions past the end of a partial group point at it).
-	__shared__ HdsHeaderSlot<kBatch, RGB> s_hdr0, s_hdr1;
-	__shared__ __attribute__((aligned(16))) float s_feat0[kRows];
-	__shared__ __attribute__((aligned(16))) float s_feat1[kRows];
-	// Per wave: the batch slots of its box-hits in list order, then kBatch (the zero row) as padding.
-	__shared__ __attribute__((aligned(16))) int s_hit[4][kBatch + kGroup];
+	// Hits in list order: mean and conic, and the gaussian and its place in the tile's list.
+	__shared__ hds_f32x4 s_mean_ab[kHits];
+	__shared__ hds_f32x2 s_c_op[kHits];
+	__shared__ int s_gid[kHits], s_idx[kHits];
+	// Feature rows and colours (16 reds, greens, blues) of the group; at the end, 32 channels of 32 pixels of the image.
+	constexpr int kChunk = 32 * 32;
+	constexpr int kFeat = S == 0 ? 4 : kGroup * S < kChunk ? kChunk : kGroup * S;
+	__shared__ __attribute__((aligned(16))) float s_feat[kFeat];
+	__shared__ __attribute__((aligned(16))) float s_rgb[RGB ? 3 * kGroup : 4];
 
-	const int tile = hds_xcd_tile(blockIdx.x, a.tiles_x, a.num_tiles);
-	if (tile < 0) return;
-	// hds_render_clear: every (tile, slice) work-group zeroes one contiguous share of the caller's
-	// range before its walk. The walk leaves most of the HBM bandwidth unused, so the 16-byte stores
-	// drain beside it instead of in a fill launch of their own; non-temporal, so the zeros do not
-	// push the walk's feature rows out of L2 (render 1.68 -> 1.61 ms at 4M gaussians, C = 256).
-	if (a.clear4 > 0) {
-		typedef float f32x4v __attribute__((ext_vector_type(4)));
-		const int64_t parts = (int64_t)a.num_tiles * gridDim.y;
-		const int64_t per = (a.clear4 + parts - 1) / parts;
-		const int64_t begin = ((int64_t)tile * gridDim.y + blockIdx.y) * per;
-		const int64_t end = min(a.clear4, begin + per);
-		f32x4v* const clear = reinterpret_cast<f32x4v*>(a.clear);
-		for (int64_t e = begin + threadIdx.x; e < end; e += blockDim.x)
-			__builtin_nontemporal_store((f32x4v){0.0f, 0.0f, 0.0f, 0.0f}, clear + e);
-	}
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+	const int block = hds_xcd_block(blockIdx.x, a.tiles_x, a.num_tiles);
+	const int lane = threadIdx.x;
+	clear_share(a, lane);
+	if (block < 0) return;
 	const int slice = blockIdx.y;
-	const int tx0 = (tile % a.tiles_x) * HDS_TILE, ty0 = (tile / a.tiles_x) * HDS_TILE;
-	const int wx0 = tx0 + (wave & 1) * 8, wy0 = ty0 + (wave >> 1) * 8;
+	const int tile = block >> 2;
+	const int wx0 = (tile % a.tiles_x) * HDS_TILE + (block & 1) * 8, wy0 = (tile / a.tiles_x) * HDS_TILE + (block >> 1 & 1) * 8;
 	const int px = wx0 + (lane & 7), py = wy0 + (lane >> 3);
 	const bool inside = px < a.width && py < a.height;
 	const float fx = (float)px + 0.5f, fy = (float)py + 0.5f;
 	const float rx0 = (float)wx0 + 0.5f, rx1 = (float)wx0 + 7.5f;
 	const float ry0 = (float)wy0 + 0.5f, ry1 = (float)wy0 + 7.5f;
 	const int2 range = a.ranges[tile];
-	const int num = range.y - range.x;
-	const int num_batches = (num + kBatch - 1) / kBatch;
 	const int c0 = slice * S;
-	auto batch_count = [&](int b) { return b < num_batches ? min(kBatch, num - b * kBatch) : 0; };
 
-	Pixel st{1.0f, !inside, 0, 0.0f, 0.0f, 0.0f};
+	Pixel st{1.0f, inside ? HDS_MIN_ALPHA : kDone, 0, 0.0f, 0.0f, 0.0f};
 	hds_f32x16 acc[2][kNcb];
 #pragma unroll
 	for (int m = 0; m < 2; m++)
 #pragma unroll
 		for (int c = 0; c < kNcb; c++) acc[m][c] = hds_f32x16{};
 
-	if (num_batches == 0) goto write_out;
-	{
-		// Prologue: gids of batches 0 and 1, then batch 0 staged synchronously.
-		if constexpr (S > 0)
-			for (int i = tid; i < S; i += blockDim.x) s_feat0[kBatch * S + i] = s_feat1[kBatch * S + i] = 0.0f;
-		const int cnt0 = batch_count(0), cnt1 = batch_count(1);
-		if (tid < cnt0) s_gid[0][tid] = a.values[range.x + tid];
-		if (tid < cnt1) s_gid[1][tid] = a.values[range.x + kBatch + tid];
-		__syncthreads();
-		hds_stage_headers_async<kBatch, RGB>(s_hdr0, a.means2D, a.conic4, a.color_op4, s_gid[0], cnt0, tid);
-		if constexpr (S > 0)
-			hds_stage_rows_async<S, false, kBatch>(s_feat0, a.features, a.channels, c0, s_gid[0], cnt0, tid);
-		hds_wait_vmem();
-		__syncthreads();
-	}
-
-	{
-		// One batch: stage b+1, read the gids of b+2, walk b. Returns true when every pixel is done.
-		auto step = [&](int b, const HdsHeaderSlot<kBatch, RGB>& h, const float* feat,
-						HdsHeaderSlot<kBatch, RGB>& h_next, float* feat_next) -> bool {
-			const int cnt = batch_count(b), cnt1 = batch_count(b + 1), cnt2 = batch_count(b + 2);
-			int g2 = 0;
-			if (tid < cnt2) g2 = a.values[range.x + (b + 2) * kBatch + tid];
-			const int* gid_next = s_gid[(b + 1) % 3];
-			if (cnt1 > 0) {
-				hds_stage_headers_async<kBatch, RGB>(h_next, a.means2D, a.conic4, a.color_op4, gid_next, cnt1, tid);
-				if constexpr (S > 0)
-					hds_stage_rows_async<S, false, kBatch>(feat_next, a.features, a.channels, c0, gid_next, cnt1, tid);
+	const int num = hds_ballot(inside) != 0 ? range.y - range.x : 0;
+	if (num > 0) {
+		const int* const values = a.values + range.x;
+		// The next batch (entries pos .. pos + 63, its records in registers) and the gids of the one after.
+		int pos = 0, gid = 0, gid_after = 0;
+		float2 mean = make_float2(0.0f, 0.0f);
+		float4 conic = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+		auto read_records = [&]() {
+			if (pos + lane < num) {
+				mean = a.means2D[gid];
+				conic = a.conic4[gid];
 			}
-
-			if (hds_ballot(!st.done) != 0) {
-				const int batch = b * kBatch;
-				bool box_hit = false;
-				if (lane < cnt) {
-					box_hit = hds_block_reach(make_float2(h.mx[lane], h.my[lane]), h.conic[lane], rx0, rx1, ry0, ry1);
-				}
-				const uint64_t hits = hds_ballot(box_hit);
-				const int total = __builtin_popcountll(hits);
-				// List the hits once per batch: hit j goes to position rank(j); positions up to the
-				// next multiple of kGroup past the last hit point at the zero row.
-				int* hit_slot = s_hit[wave];
-				if (box_hit) hit_slot[hds_rank_below(hits)] = lane;
-				if (lane >= total && lane < ((total + kGroup - 1) & ~(kGroup - 1))) hit_slot[lane] = kBatch;
-				hds_wave_fence();
-				for (int g0 = 0; g0 < total; g0 += kGroup) {
-					// The next group: up to 16 box-hits in list order; missing positions use the zero row.
-					const int count = min(kGroup, total - g0);
-					int slot[kGroup];
-#pragma unroll
-					for (int q4 = 0; q4 < kGroup; q4 += 4) {
-						const int4 v = *reinterpret_cast<const int4*>(hit_slot + g0 + q4);
-						slot[q4] = v.x;
-						slot[q4 + 1] = v.y;
-						slot[q4 + 2] = v.z;
-						slot[q4 + 3] = v.w;
-					}
-					float w[kGroup];
-#pragma unroll
-					for (int q0 = 0; q0 < kGroup; q0 += kIlp) {
-						if (q0 >= count) {
-							// Past the group's last hit (wave-uniform): nothing to evaluate.
-#pragma unroll
-							for (int u = 0; u < kIlp; u++) w[q0 + u] = 0.0f;
-							continue;
-						}
-						float alpha[kIlp];
-						float4 col[kIlp];
-#pragma unroll
-						for (int u = 0; u < kIlp; u++) {
-							const int sl = min(slot[q0 + u], kBatch - 1);
-							float G, dx, dy;
-							alpha[u] = fminf(HDS_MAX_ALPHA, hds_raw_alpha(fx, fy, make_float2(h.mx[sl], h.my[sl]),
-																		  h.conic[sl], G, dx, dy));
-							// Read with the geometry: a read under the blend branch would stall on LDS latency.
-							if constexpr (RGB) col[u] = h.color[sl];
-						}
-#pragma unroll
-						for (int u = 0; u < kIlp; u++) {
-							const int q = q0 + u;
-							w[q] = 0.0f;
-							if (q < count && !st.done && alpha[u] >= HDS_MIN_ALPHA) {
-								const float test_T = st.T * (1.0f - alpha[u]);
-								if (test_T < HDS_MIN_TRANSMITTANCE) {
-									st.done = true;
-								} else {
-									w[q] = alpha[u] * st.T;
-									if constexpr (RGB) {
-										// fmaf as the oracle does: the RGB image is bit-exact.
-										st.r = fmaf(w[q], col[u].x, st.r);
-										st.g = fmaf(w[q], col[u].y, st.g);
-										st.b = fmaf(w[q], col[u].z, st.b);
-									}
-									st.T = test_T;
-									st.last = batch + slot[q] + 1;
-								}
-							}
-						}
-					}
-					if constexpr (S > 0) {
-						uint32_t w_hi[8], w_lo[8];
-#pragma unroll
-						for (int i = 0; i < 8; i++) hds_split_pair(w[2 * i], w[2 * i + 1], w_hi[i], w_lo[i]);
-						flush_group<S>(acc, w_hi, w_lo, slot, feat, lane);
-					}
-					if (hds_ballot(!st.done) == 0) break;
-				}
-			}
-
-			if (tid < cnt2) s_gid[(b + 2) % 3][tid] = g2;
-			hds_wait_vmem();
-			return __syncthreads_count(st.done) == (int)blockDim.x;
+			if (pos + kBatch + lane < num) gid_after = values[pos + kBatch + lane];
 		};
-		for (int b = 0; b < num_batches; b += 2) {
-			if (step(b, s_hdr0, s_feat0, s_hdr1, s_feat1) || b + 1 >= num_batches) break;
-			if (step(b + 1, s_hdr1, s_feat1, s_hdr0, s_feat0)) break;
+		if (lane < num) gid = values[lane];
+		read_records();
+
+		int head = 0, count = 0;  // pending hits: list positions head .. head + count - 1
+		// Tests batches until `want` hits are pending or the list ends.
+		auto top_up = [&](int want) {
+			const int lane = (int)hds_opaque(threadIdx.x);
+			while (count < want && pos < num) {
+				const bool hit = pos + lane < num && hds_block_reach(mean, conic, rx0, rx1, ry0, ry1);
+				const uint64_t hits = hds_ballot(hit);
+				if (hits != 0) {
+					if (head > 0) {
+						// At most 31 hits are left: to the front.
+						if (lane < count) {
+							const hds_f32x4 m = s_mean_ab[head + lane];
+							const hds_f32x2 c = s_c_op[head + lane];
+							const int g = s_gid[head + lane], i = s_idx[head + lane];
+							s_mean_ab[lane] = m;
+							s_c_op[lane] = c;
+							s_gid[lane] = g;
+							s_idx[lane] = i;
+						}
+						hds_wave_fence();
+						head = 0;
+					}
+					if (hit) {
+						const int at = count + hds_rank_below(hits);
+						s_mean_ab[at] = hds_f32x4{mean.x, mean.y, conic.x, conic.y};
+						s_c_op[at] = hds_f32x2{conic.z, conic.w};
+						s_gid[at] = gid;
+						s_idx[at] = pos + lane;
+					}
+					count += __builtin_popcountll(hits);
+				}
+				pos += kBatch;
+				gid = gid_after;
+				read_records();
+			}
+			hds_wave_fence();
+		};
+		for (;;) {
+			top_up(kGroup);
+			const int n = min(count, kGroup), first = head;
+			if (n == 0) break;
+			head += n;
+			count -= n;
+			stage_group<S, RGB>(s_feat, s_rgb, a, s_gid, first, n, c0);
+			float w[kGroup];
+			int last = -1;
+#pragma unroll
+			for (int q0 = 0; q0 < kGroup; q0 += kIlp) {
+				// The records of four hits, then their four alphas, then the chain through T: left alone, the
+				// compiler takes the hits one by one, each behind its own LDS read and the alpha before it.
+				hds_f32x4 ma[kIlp];
+				hds_f32x2 co[kIlp];
+				float alpha[kIlp];
+#pragma unroll
+				for (int u = 0; u < kIlp; u++) {
+					ma[u] = s_mean_ab[first + q0 + u];
+					co[u] = s_c_op[first + q0 + u];
+				}
+				asm volatile("" : "+v"(ma[0]), "+v"(ma[1]), "+v"(ma[2]), "+v"(ma[3]), "+v"(co[0]), "+v"(co[1]), "+v"(co[2]),
+							 "+v"(co[3]));
+#pragma unroll
+				for (int u = 0; u < kIlp; u++) {
+					float G, dx, dy;
+					alpha[u] = fminf(HDS_MAX_ALPHA, hds_raw_alpha(fx, fy, make_float2(ma[u].x, ma[u].y),
+																  make_float4(ma[u].z, ma[u].w, co[u].x, co[u].y), G, dx, dy));
+				}
+				asm volatile("" : "+v"(alpha[0]), "+v"(alpha[1]), "+v"(alpha[2]), "+v"(alpha[3]));
+				bool blends[kIlp];
+				float T[kIlp + 1];
+				T[0] = st.T;
+#pragma unroll
+				for (int u = 0; u < kIlp; u++) {
+					blends[u] = q0 + u < n && alpha[u] >= st.reach;
+					alpha[u] = blends[u] ? alpha[u] : 0.0f;
+					w[q0 + u] = alpha[u] * T[u];
+					T[u + 1] = T[u] * (1.0f - alpha[u]);
+				}
+				if (hds_ballot(T[kIlp] < HDS_MIN_TRANSMITTANCE) != 0) {
+					// Some pixel stops here, before the gaussian that takes its T below the limit.
+					st.reach = T[kIlp] < HDS_MIN_TRANSMITTANCE ? kDone : st.reach;
+					float kept = T[0];
+#pragma unroll
+					for (int u = 0; u < kIlp; u++) {
+						const bool below = T[u + 1] < HDS_MIN_TRANSMITTANCE;
+						blends[u] = blends[u] && !below;
+						w[q0 + u] = below ? 0.0f : w[q0 + u];
+						kept = below ? kept : T[u + 1];
+					}
+					T[kIlp] = kept;
+				}
+				st.T = T[kIlp];
+#pragma unroll
+				for (int u = 0; u < kIlp; u++) last = blends[u] ? q0 + u : last;
+			}
+			if (last >= 0) st.n_contrib = s_idx[first + last] + 1;
+			wait_vmem();
+			if constexpr (RGB) {
+				// fmaf as the oracle does: the RGB image is bit-exact. A colour that is not finite would turn the 0 of
+				// a gaussian that does not blend into NaN.
+				const float c = s_rgb[min(lane, 3 * kGroup - 1)];
+				const bool any_odd = hds_ballot(!(c - c == 0.0f)) != 0;
+#pragma unroll
+				for (int q0 = 0; q0 < kGroup; q0 += 4) {
+					hds_f32x4 color[3];
+#pragma unroll
+					for (int k = 0; k < 3; k++) color[k] = *reinterpret_cast<const hds_f32x4*>(s_rgb + k * kGroup + q0);
+					if (__builtin_expect(any_odd, 0)) {
+#pragma unroll
+						for (int u = 0; u < 4; u++) {
+							if (!(w[q0 + u] > 0.0f)) continue;
+							st.r = fmaf(w[q0 + u], color[0][u], st.r);
+							st.g = fmaf(w[q0 + u], color[1][u], st.g);
+							st.b = fmaf(w[q0 + u], color[2][u], st.b);
+						}
+						asm volatile("" : "+v"(st.r));  // a branch, not three selects per hit
+					} else {
+#pragma unroll
+						for (int u = 0; u < 4; u++) {
+							st.r = fmaf(w[q0 + u], color[0][u], st.r);
+							st.g = fmaf(w[q0 + u], color[1][u], st.g);
+							st.b = fmaf(w[q0 + u], color[2][u], st.b);
+						}
+					}
+				}
+			}
+			if constexpr (S > 0) {
+				uint32_t w_hi[8], w_lo[8];
+#pragma unroll
+				for (int i = 0; i < 8; i++) hds_split_pair(w[2 * i], w[2 * i + 1], w_hi[i], w_lo[i]);
+				flush_group<S>(acc, w_hi, w_lo, s_feat, lane);
+			}
+			if (hds_ballot(st.reach < kDone) == 0) break;
 		}
 	}
 
-write_out:
 	if (inside && slice == 0) {
 		const int64_t pix = (int64_t)py * a.width + px;
 		if constexpr (RGB) {
@@ -287,32 +370,41 @@ write_out:
 			a.image[pix * 3 + 2] = fmaf(st.T, a.background[2], st.b);
 		}
 		a.final_T[pix] = st.T;
-		a.n_contrib[pix] = st.last;
+		a.n_contrib[pix] = st.n_contrib;
 	}
 	if constexpr (S > 0) {
-		// D of a 32x32 tile: lane holds pixel 32m + lane % 32 and, for each group g of four
-		// accumulators, channels 8g + 4 (lane / 32) + 0..3.
+		// D of a 32x32 tile: lane holds pixel 32m + lane % 32 and, for each group g of four accumulators, channels
+		// 8g + 4 (lane / 32) + 0..3. By way of LDS, 32 channels of 32 pixels at a time, to whole lines: eight lanes
+		// store a pixel's 128 bytes. The 16-byte pieces of a pixel are permuted by its number, against bank conflicts.
+		hds_f32x4* const piece = reinterpret_cast<hds_f32x4*>(s_feat);
 #pragma unroll
-		for (int m = 0; m < 2; m++) {
-			const int p = 32 * m + (lane & 31);
-			const int x = wx0 + (p & 7), y = wy0 + (p >> 3);
-			if (x >= a.width || y >= a.height) continue;
-			float* dst = a.feature_image + ((int64_t)y * a.width + x) * a.channels + c0 + 4 * (lane >> 5);
+		for (int c = 0; c < kNcb; c++)
 #pragma unroll
-			for (int c = 0; c < kNcb; c++)
+			for (int m = 0; m < 2; m++) {
+				const hds_f32x16 v = acc[m][c];
+				hds_f32x4* const half = piece + (kFeat >= 2 * kChunk ? kChunk / 4 * m : 0);
+				hds_wave_fence();
 #pragma unroll
-				for (int g = 0; g < 4; g++) {
-					const hds_f32x16 v = acc[m][c];
-					*reinterpret_cast<float4*>(dst + 32 * c + 8 * g) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+				for (int g = 0; g < 4; g++)
+					half[8 * (lane & 31) + ((2 * g + (lane >> 5)) ^ (lane & 7))] = hds_f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+				hds_wave_fence();
+#pragma unroll
+				for (int i = 0; i < 4; i++) {
+					const int p = 8 * i + (lane >> 3);
+					const int x = wx0 + (p & 7), y = wy0 + 4 * m + (p >> 3);
+					const hds_f32x4 out = half[8 * p + ((lane & 7) ^ (p & 7))];
+					if (x < a.width && y < a.height)
+						__builtin_nontemporal_store(out, reinterpret_cast<hds_f32x4*>(a.feature_image + ((int64_t)y * a.width + x) * a.channels +
+																					  c0 + 32 * c) + (lane & 7));
 				}
-		}
+			}
 	}
 }
 
 template <int S, bool RGB>
 int launch(const RenderArgs& a, int num_tiles, int slices, hipStream_t s) {
 	HdsKernelTimer timer1("render_forward_kernel", s);
-	render_forward_kernel<S, RGB><<<dim3(hds_xcd_grid(a.tiles_x, num_tiles), (unsigned)slices), 256, 0, s>>>(a);
+	render_forward_kernel<S, RGB><<<dim3(hds_xcd_block_grid(a.tiles_x, num_tiles), (unsigned)slices), 64, 0, s>>>(a);
 	timer1.stop();
 	return hds_check_launch(RGB ? (S > 0 ? "render_rgb_features" : "render_rgb") : "render_features", s);
 }

@@ -121,7 +121,9 @@ def test_a_non_finite_pixel_gradient_reaches_only_the_gaussians_it_sees(value):
     """One pixel's dL/dRGB is not finite: the geometry gradients of gaussians that do not touch that pixel's block
     are the oracle's, and those of gaussians in the block that do not contribute to the pixel stay finite."""
     width = height = 32
-    inputs = flat_scene([[3.5, 3.5], [6.5, 6.5], [20.0, 20.0]], [1.0, 2.0, 3.0], [0.5, 0.5, 1.5], [0.8, 0.7, 0.6], device=DEV)
+    # The third gaussian reaches 0.5 sqrt(2 ln(255 * 0.6)) = 1.6 pixels, so one block: its gradient is a single row, the
+    # same bits in both runs (the rows of several tiles are summed in the order they were counted in).
+    inputs = flat_scene([[3.5, 3.5], [6.5, 6.5], [20.0, 20.0]], [1.0, 2.0, 3.0], [0.5, 0.5, 0.5], [0.8, 0.7, 0.6], device=DEV)
 
     def poison(gi, gf):
         gi = gi.clone()
