@@ -1,7 +1,8 @@
 // Blend backward through per-block gaussian lists and stored gradient rows (hds_render_backward_rows).
 //
-// 1. backward_lists_kernel: per tile, the gaussians that can reach each of its four 8x8 pixel blocks (up to
-//    the block's deepest contributor), deepest first, as one list per block; every (gaussian, block) hit
+// 1. backward_lists_kernel: per tile, the gaussians that blend into each of its four 8x8 pixel blocks (from the
+//    render's marks; without marks, those that can reach the block, up to its deepest contributor), deepest first,
+//    as one list per block; every (gaussian, block) hit
 //    gets the next row number of its gaussian.
 // 2. backward_base_kernel: one contiguous range of rows per gaussian.
 // 3. backward_geometry_kernel: the replay. Work-group = one block x slice of S channels, two waves; it walks
@@ -35,8 +36,8 @@
 // stores plus 0.17 ms as loads.
 //
 // Measured at 1.18M gaussians, 979x546, against the two kernels of hds_render_backward (lane = pixel, a
-// serial chain per gaussian, atomics; side by side): C = 128 lists 0.11 + replay 0.81 + sums 0.45 ms for 1.68,
-// RGB alone 0.11 + 0.36 + 0.07 for 0.66, C = 512 5.0 for 6.4; 4M gaussians at 1920x1080, C = 256: 2.7 for 4.2. The
+// serial chain per gaussian, atomics; side by side): C = 128 lists 0.08 + replay 0.74 + sums 0.42 ms for 1.68,
+// RGB alone 0.08 + 0.32 + 0.06 for 0.66, C = 512 4.5 for 6.4; 4M gaussians at 1920x1080, C = 256: 2.6 for 4.2. The
 // replay issues 1,290 VALU instructions per group (0.36 ms), 106 MFMAs (0.11 ms), and moves 1.3 GB of feature
 // rows in and 1.5 GB of gradient rows out; it runs two waves per SIMD (250 VGPRs, 40 KB of LDS per block).
 #include <algorithm>
@@ -91,6 +92,7 @@ struct BackwardArgs {
 	const float* background;
 	const float* final_T;
 	const int* n_contrib;
+	const uint8_t* contributes;  // the render's marks (hds_render_contributes), or null
 	const float* grad_image;
 	const float* features;
 	const float* grad_feature_image;
@@ -103,10 +105,14 @@ struct BackwardArgs {
 	Rows rows;
 };
 
-// One work-group per tile. A thread tests one list entry per step against the tile's four blocks (their
-// tests share most of the arithmetic, and every record is gathered once); the records of the next step are
-// in flight meanwhile. Bound by latency and the one returning atomic per (gaussian, tile).
+// One work-group per tile, a list entry per thread and step, what the next step needs in flight meanwhile. With the
+// render's marks (kMarked) a block's list holds exactly what blends into it; without them, what can reach it: a
+// thread tests its entry against the tile's four blocks (their tests share most of the arithmetic, and every
+// record is gathered once). Bound by latency and the one returning atomic per (gaussian, tile). At 1.18M
+// gaussians, 979x546, C = 128 marks take 0.020 ms of the render and save 0.026 here (0.108 -> 0.082), 0.065 of the
+// geometry and 0.036 of the sums, which have a tenth fewer rows.
 constexpr int kListThreads = 256;
+template <bool kMarked>
 __global__ __launch_bounds__(kListThreads) void backward_lists_kernel(const BackwardArgs a) {
 	__shared__ int s_last[4];
 	__shared__ int s_count[2][4][4];  // per step parity: [wave][block]
@@ -131,26 +137,36 @@ __global__ __launch_bounds__(kListThreads) void backward_lists_kernel(const Back
 	int gid = 0, later = 0;
 	float2 mean = make_float2(0.0f, 0.0f);
 	float4 conic = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	uint8_t mark[4] = {0, 0, 0, 0};
+	// The records or marks of entry e (gaussian gid).
+	auto fetch = [&](int e) {
+		if constexpr (kMarked) {
+#pragma unroll
+			for (int b = 0; b < 4; b++) mark[b] = a.contributes[out + (int64_t)b * len + max(e, 0)];
+		} else {
+			mean = a.means2D[gid];
+			conic = a.conic4[gid];
+		}
+	};
 	if (num > 0) {
 		gid = list[max(num - 1 - tid, 0)];
 		later = list[max(num - 1 - kListThreads - tid, 0)];
-		mean = a.means2D[gid];
-		conic = a.conic4[gid];
+		fetch(num - 1 - tid);
 	}
 	for (int step = 0; step * kListThreads < num; step++) {
 		const int e = num - 1 - step * kListThreads - tid, g = gid;
 		const float2 m = mean;
 		const float4 c = conic;
+		const uint8_t marked[4] = {mark[0], mark[1], mark[2], mark[3]};
 		gid = later;
-		mean = a.means2D[gid];
-		conic = a.conic4[gid];
+		fetch(e - kListThreads);
 		later = list[max(e - 2 * kListThreads, 0)];
 		uint64_t hits[4];
 		int mask = 0;
 #pragma unroll
 		for (int b = 0; b < 4; b++) {
 			const float x0 = (float)(tx0 + (b & 1) * 8) + 0.5f, y0 = (float)(ty0 + (b >> 1) * 8) + 0.5f;
-			const bool hit = e >= 0 && e < last[b] && hds_block_reach(m, c, x0, x0 + 7.0f, y0, y0 + 7.0f);
+			const bool hit = e >= 0 && e < last[b] && (kMarked ? marked[b] != 0 : hds_block_reach(m, c, x0, x0 + 7.0f, y0, y0 + 7.0f));
 			hits[b] = hds_ballot(hit);
 			mask |= (int)hit << b;
 		}
@@ -957,8 +973,8 @@ extern "C" size_t hds_render_backward_workspace_bytes(int64_t n, int width, int 
 					 channels > 0 ? channels / slice_width : 1).bytes;
 }
 
-extern "C" int hds_render_backward_rows(HDS_BACKWARD_ARGS, int zeroed, int64_t row_capacity, void* workspace,
-										size_t workspace_bytes, hds_stream_t stream) {
+extern "C" int hds_render_backward_rows(HDS_BACKWARD_ARGS, int zeroed, const uint8_t* contributes, int64_t row_capacity,
+										void* workspace, size_t workspace_bytes, hds_stream_t stream) {
 	HDS_REQUIRE(width > 0 && height > 0, "render_backward: image size %dx%d must be positive", width, height);
 	HDS_REQUIRE(n >= 0, "render_backward: negative gaussian count");
 	HDS_REQUIRE(tile_ranges && final_T && n_contrib && (n == 0 || (grad_means2D && grad_conics && grad_opacities)),
@@ -1031,6 +1047,7 @@ extern "C" int hds_render_backward_rows(HDS_BACKWARD_ARGS, int zeroed, int64_t r
 	a.background = background;
 	a.final_T = final_T;
 	a.n_contrib = n_contrib;
+	a.contributes = contributes;
 	a.grad_image = grad_image;
 	a.features = features;
 	a.grad_feature_image = grad_feature_image;
@@ -1049,7 +1066,10 @@ extern "C" int hds_render_backward_rows(HDS_BACKWARD_ARGS, int zeroed, int64_t r
 				  slices};
 	{
 		HdsKernelTimer timer("backward_lists_kernel", s);
-		backward_lists_kernel<<<(unsigned)num_tiles, kListThreads, 0, s>>>(a);
+		if (contributes)
+			backward_lists_kernel<true><<<(unsigned)num_tiles, kListThreads, 0, s>>>(a);
+		else
+			backward_lists_kernel<false><<<(unsigned)num_tiles, kListThreads, 0, s>>>(a);
 		timer.stop();
 		HDS_LAUNCH_CHECK("backward_lists", s);
 	}

@@ -61,6 +61,7 @@ struct RenderArgs {
 	float* feature_image;
 	float4* clear;   // hds_render_clear's range (clear4 16-byte words), or null
 	int64_t clear4;
+	uint8_t* contributes;  // hds_render_contributes' marks, or null
 };
 
 // Feature rows of a group in LDS, S floats each, in the order of their copy: wave instruction i brings 1 KB, in its
@@ -211,6 +212,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2
 		for (int c = 0; c < kNcb; c++) acc[m][c] = hds_f32x16{};
 
 	const int num = hds_ballot(inside) != 0 ? range.y - range.x : 0;
+	// This block's marks, one byte per list entry: 0 from the test of an entry that cannot reach the block, the others
+	// from the group they are blended in.
+	uint8_t* const marks = a.contributes && slice == 0 ? a.contributes + 4 * (int64_t)range.x + (int64_t)(block & 3) * num : nullptr;
 	if (num > 0) {
 		const int* const values = a.values + range.x;
 		// The next batch (entries pos .. pos + 63, its records in registers) and the gids of the one after.
@@ -234,6 +238,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2
 			while (count < want && pos < num) {
 				const bool hit = pos + lane < num && hds_block_reach(mean, conic, rx0, rx1, ry0, ry1);
 				const uint64_t hits = hds_ballot(hit);
+				if (marks && !hit && pos + lane < num) marks[pos + lane] = 0;
 				if (hits != 0) {
 					if (head > 0) {
 						// At most 31 hits are left: to the front.
@@ -273,6 +278,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2
 			stage_group<S, RGB>(s_feat, s_rgb, a, s_gid, first, n, c0);
 			float w[kGroup];
 			int last = -1;
+			uint32_t contribute = 0;  // bit q: hit q blends into some pixel
 #pragma unroll
 			for (int q0 = 0; q0 < kGroup; q0 += kIlp) {
 				// The records of four hits, then their four alphas, then the chain through T: left alone, the
@@ -319,10 +325,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S >= 128 ? 2
 				}
 				st.T = T[kIlp];
 #pragma unroll
-				for (int u = 0; u < kIlp; u++) last = blends[u] ? q0 + u : last;
+				for (int u = 0; u < kIlp; u++) {
+					last = blends[u] ? q0 + u : last;
+					contribute |= hds_ballot(blends[u]) != 0 ? 1u << (q0 + u) : 0u;
+				}
 			}
 			if (last >= 0) st.n_contrib = s_idx[first + last] + 1;
 			wait_vmem();
+			if (marks && lane < n) marks[s_idx[first + lane]] = (uint8_t)(contribute >> lane & 1u);
 			if constexpr (RGB) {
 				// fmaf as the oracle does: the RGB image is bit-exact. A colour that is not finite would turn the 0 of
 				// a gaussian that does not blend into NaN.
@@ -414,7 +424,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int render(int width, int height, int channels, const int32_t* tile_ranges, const int32_t* values_sorted,
 		   int64_t num_pairs, const float* means2D, const float* conic4, const float* color_opacity4,
 		   const float* background, const float* features, float* image, float* final_T, int32_t* n_contrib,
-		   float* feature_image, float* clear, int64_t clear_count, hds_stream_t stream) {
+		   float* feature_image, float* clear, int64_t clear_count, uint8_t* contributes, hds_stream_t stream) {
 	HDS_REQUIRE(clear_count >= 0, "render_clear: negative clear count");
 	HDS_REQUIRE(clear_count == 0 || (clear && aligned16(clear) && clear_count % 4 == 0),
 				"render_clear: needs a 16-byte aligned range of a multiple of 4 floats");
@@ -451,7 +461,8 @@ int render(int width, int height, int channels, const int32_t* tile_ranges, cons
 				 n_contrib,
 				 feature_image,
 				 reinterpret_cast<float4*>(clear),
-				 clear_count / 4};
+				 clear_count / 4,
+				 contributes};
 	hipStream_t s = (hipStream_t)stream;
 	if (!feats) {
 		HDS_REQUIRE(rgb, "render: nothing to render (no image and no features)");
@@ -480,7 +491,7 @@ extern "C" int hds_render(int64_t n, int width, int height, int channels, const 
 						  float* final_T, int32_t* n_contrib, float* feature_image, hds_stream_t stream) {
 	(void)n;
 	return render(width, height, channels, tile_ranges, values_sorted, num_pairs, means2D, conic4, color_opacity4,
-				  background, features, image, final_T, n_contrib, feature_image, nullptr, 0, stream);
+				  background, features, image, final_T, n_contrib, feature_image, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int hds_render_clear(int64_t n, int width, int height, int channels, const int32_t* tile_ranges,
@@ -490,5 +501,17 @@ extern "C" int hds_render_clear(int64_t n, int width, int height, int channels, 
 								float* feature_image, float* clear, int64_t clear_count, hds_stream_t stream) {
 	(void)n;
 	return render(width, height, channels, tile_ranges, values_sorted, num_pairs, means2D, conic4, color_opacity4,
-				  background, features, image, final_T, n_contrib, feature_image, clear, clear_count, stream);
+				  background, features, image, final_T, n_contrib, feature_image, clear, clear_count, nullptr, stream);
+}
+
+extern "C" int hds_render_contributes(int64_t n, int width, int height, int channels, const int32_t* tile_ranges,
+									  const int32_t* values_sorted, int64_t num_pairs, const float* means2D,
+									  const float* conic4, const float* color_opacity4, const float* background,
+									  const float* features, float* image, float* final_T, int32_t* n_contrib,
+									  float* feature_image, float* clear, int64_t clear_count, uint8_t* contributes,
+									  hds_stream_t stream) {
+	(void)n;
+	HDS_REQUIRE(contributes || num_pairs == 0, "render_contributes: null marks");
+	return render(width, height, channels, tile_ranges, values_sorted, num_pairs, means2D, conic4, color_opacity4,
+				  background, features, image, final_T, n_contrib, feature_image, clear, clear_count, contributes, stream);
 }

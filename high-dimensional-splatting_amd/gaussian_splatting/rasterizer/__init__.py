@@ -68,17 +68,27 @@ class RasterizeGaussians(torch.autograd.Function):
             features = features.contiguous()
         background = background.contiguous()
         conic, color_opacity, tile_ranges = bins.conic4, bins.color_opacity4, bins.tile_ranges
+        # What contributes to each block, for a backward to come: a byte per (block, pair).
+        marks = grad_enabled and any(ctx.needs_input_grad[i] for i in (0, 3, 4, 5, 7))
+
+        def contributes_buffer():
+            return (torch.empty(4 * bins.values.numel(), device=means2D.device, dtype=torch.uint8) if marks
+                    and bins.values.numel() else None)
+
+        contributes = contributes_buffer()
         image, feature_image, final_T, n_contrib = ext.render(
             means2D, conic, color_opacity, bins.values, tile_ranges, width, height, background, features,
-            clear=clear)
+            clear=clear, contributes=contributes)
         # A render again after a rebin: the buffers were already cleared (on this stream) by the first.
         if ext.resolve(bins):
+            contributes = contributes_buffer()
             image, feature_image, final_T, n_contrib = ext.render(
-                means2D, conic, color_opacity, bins.values, tile_ranges, width, height, background, features)
+                means2D, conic, color_opacity, bins.values, tile_ranges, width, height, background, features,
+                contributes=contributes)
         values_sorted = bins.values
         ctx.image_size = (width, height)
         ctx.save_for_backward(means2D, conic, color_opacity, values_sorted, tile_ranges, final_T, n_contrib,
-                              background, features)
+                              background, features, contributes)
         if features is None:
             return image
         return image, feature_image
@@ -91,8 +101,8 @@ class RasterizeGaussians(torch.autograd.Function):
             Gradients for means2D, conics, colors, opacities and features; None for depths, radii,
             background and the image size.
         """
-        means2D, conic, color_opacity, values_sorted, tile_ranges, final_T, n_contrib, background, features = (
-            ctx.saved_tensors)
+        (means2D, conic, color_opacity, values_sorted, tile_ranges, final_T, n_contrib, background, features,
+         contributes) = ctx.saved_tensors
         width, height = ctx.image_size
         # Frozen features still shape the geometry gradients, so the feature term runs whenever any of
         # means2D, conics, opacities or features needs a gradient (rasterizer/__init__.py:150-152).
@@ -107,7 +117,8 @@ class RasterizeGaussians(torch.autograd.Function):
                 features=features if feature_term else None,
                 grad_feature_image=grad_features.contiguous() if feature_term else None,
                 slice_width=(FEATURE_SLICE_WIDTH or default_slice_width(features.shape[1])) if feature_term else None,
-                want_feature_grad=feature_term and ctx.needs_input_grad[7], prezeroed=ctx.prezeroed)
+                want_feature_grad=feature_term and ctx.needs_input_grad[7], prezeroed=ctx.prezeroed,
+                contributes=contributes)
         ctx.prezeroed = None
         return g_means, None, None, g_conics, g_colors, g_opac, None, g_feat, None, None, None
 

@@ -57,13 +57,16 @@ PROTOTYPES = {
                           _vp]),
     "hds_render_clear": (_i32, [_i64, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                 _vp, _vp, _i64, _vp]),
+    "hds_render_contributes": (_i32, [_i64, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                      _vp, _vp, _i64, _vp, _vp]),
     "hds_render_backward": (_i32, [_i64, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_render_backward_accumulate": (_i32, [_i64, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp,
                                               _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_render_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
     "hds_render_backward_rows": (_i32, [_i64, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp,
-                                        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _vp, _sz, _vp]),
+                                        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _sz,
+                                        _vp]),
     "hds_ssim_forward": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_ssim_backward": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "hds_densification_stats": (_i32, [_i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
@@ -531,9 +534,10 @@ class HipRasterizer:
         self._pair_capacity[dev.index] = (int(pairs * self.PAIR_HEADROOM) + 2 * chunk) // chunk * chunk
 
     def render(self, means2D, conic4, color_opacity4, values_sorted, tile_ranges, width, height, background=None,
-               features=None, rgb=True, clear=None):
+               features=None, rgb=True, clear=None, contributes=None):
         """One front-to-back tile walk (forward.cu:141-237 + features.cu:116-282). With `clear` (a float32
-        tensor from gradient_buffers), the walk's work-groups also zero it (hds_render_clear).
+        tensor from gradient_buffers), the walk's work-groups also zero it (hds_render_clear); with `contributes`
+        (uint8, four per pair), they mark there what blends into each block (hds_render_contributes).
 
         Returns (image [H,W,3] or None, feature_image [H,W,C] or None, final_T [H,W], n_contrib [H,W]).
         """
@@ -562,8 +566,15 @@ class HipRasterizer:
         if clear is not None and not (clear.is_cuda and clear.is_contiguous() and clear.dtype == torch.float32
                                       and clear.device == dev):
             raise RuntimeError("clear must be a contiguous float32 tensor on the render's device")
+        if contributes is not None and not (contributes.is_cuda and contributes.is_contiguous() and contributes.device == dev
+                                            and contributes.dtype == torch.uint8
+                                            and contributes.numel() >= 4 * values_sorted.numel()):
+            raise RuntimeError("contributes must hold four uint8 per pair on the render's device")
         with torch.cuda.device(dev):
-            if clear is None:
+            if contributes is not None:
+                self._run("render", lambda: self.lib.hds_render_contributes(
+                    *args, _ptr(clear), 0 if clear is None else clear.numel(), _ptr(contributes), _stream(dev)))
+            elif clear is None:
                 self._run("render", lambda: self.lib.hds_render(*args, _stream(dev)))
             else:
                 self._run("render", lambda: self.lib.hds_render_clear(*args, _ptr(clear), clear.numel(),
@@ -572,10 +583,11 @@ class HipRasterizer:
 
     def render_backward(self, means2D, conic4, color_opacity4, values_sorted, tile_ranges, final_T, n_contrib,
                         width, height, grad_image=None, background=None, features=None, grad_feature_image=None,
-                        slice_width=None, want_feature_grad=True, prezeroed=None):
+                        slice_width=None, want_feature_grad=True, prezeroed=None, contributes=None):
         """The blend backward (backward.cu:7-164 + features.cu:350-542): hds_render_backward_rows where its workspace
         fits, else the atomic hds_render_backward. `prezeroed` is the buffers of gradient_buffers, zeroed by
-        earlier work on the current stream (render(clear=...)), to write the gradients into.
+        earlier work on the current stream (render(clear=...)), to write the gradients into; `contributes` is the marks of
+        render(contributes=...) on the same frame.
 
         Returns (grad_means2D [N,2], grad_conics [N,3], grad_colors [N,3] or None, grad_opacities [N,1],
         grad_features [N,C] or None).
@@ -616,7 +628,7 @@ class HipRasterizer:
                                                        values_sorted.numel(), dev)
             if workspace is not None:
                 self._run("render_backward", lambda: self.lib.hds_render_backward_rows(
-                    *args, int(prezeroed is not None), rows, _ptr(workspace), workspace.numel(), _stream(dev)))
+                    *args, int(prezeroed is not None), _ptr(contributes), rows, _ptr(workspace), workspace.numel(), _stream(dev)))
             else:
                 entry = (self.lib.hds_render_backward if prezeroed is None
                          else self.lib.hds_render_backward_accumulate)

@@ -240,6 +240,16 @@ HDS_API int hds_render_clear(int64_t n, int width, int height, int channels, con
 				 const float* features, float* image, float* final_T, int32_t* n_contrib,
 				 float* feature_image, float* clear, int64_t clear_count, hds_stream_t stream);
 
+/* hds_render_clear (clear may be NULL) that also marks what contributes, for hds_render_backward_rows: byte
+ * 4 * begin + b * length + i of contributes (4 * num_pairs bytes) is 1 if entry i of a tile's list [begin, begin + length)
+ * blends into a pixel of its 8x8 block b (x half + 2 * y half), else 0. Bytes of entries past a block's
+ * deepest contributor need not be written. */
+HDS_API int hds_render_contributes(int64_t n, int width, int height, int channels, const int32_t* tile_ranges,
+				 const int32_t* values_sorted, int64_t num_pairs, const float* means2D,
+				 const float* conic4, const float* color_opacity4, const float* background,
+				 const float* features, float* image, float* final_T, int32_t* n_contrib,
+				 float* feature_image, float* clear, int64_t clear_count, uint8_t* contributes, hds_stream_t stream);
+
 /* ---- blend backward: replaces rasterize_backward (backward.cu:166-226) and
  *      rasterize_features_backward (features.cu:561-616) with one back-to-front walk ----------- */
 
@@ -273,7 +283,8 @@ HDS_API size_t hds_render_backward_workspace_bytes(int64_t n, int width, int hei
 /* hds_render_backward through a workspace: the blend's gradients of each (gaussian, 8x8 pixel block) are stored as
  * a row, and each gaussian's rows are summed by a second pass, instead of being added atomically. At most
  * row_capacity rows (up to 2^30 - 1024) are stored; the gradients of rows past that are added atomically. zeroed != 0: the
- * gradient outputs hold zeros already. The workspace (16-byte aligned, its contents do not matter) is free
+ * gradient outputs hold zeros already. contributes: the marks of the render of this frame (hds_render_contributes), or NULL,
+ * and the gaussians that can reach a block are found again. The workspace (16-byte aligned, its contents do not matter) is free
  * again when the stream has run the call. */
 HDS_API int hds_render_backward_rows(
 	int64_t n, int width, int height, int channels, int slice_width, const int32_t* tile_ranges,
@@ -281,7 +292,7 @@ HDS_API int hds_render_backward_rows(
 	const float* color_opacity4, const float* background, const float* final_T, const int32_t* n_contrib,
 	const float* grad_image, const float* features, const float* grad_feature_image, float* grad_means2D,
 	float* grad_conics, float* grad_colors, float* grad_opacities, float* grad_features, int zeroed,
-	int64_t row_capacity, void* workspace, size_t workspace_bytes, hds_stream_t stream);
+	const uint8_t* contributes, int64_t row_capacity, void* workspace, size_t workspace_bytes, hds_stream_t stream);
 
 /* Zeroes `count` floats at p (16-byte aligned, count a multiple of 4) on `stream` with at most
  * `max_workgroups` work-groups of 256 threads (0: as many as fill the device), so that a large fill

@@ -136,3 +136,44 @@ def test_a_non_finite_pixel_gradient_reaches_only_the_gaussians_it_sees(value):
     for k in (0, 1, 3):
         assert np.isfinite(got[k][1:]).all(), NAMES[k]
         np.testing.assert_array_equal(got[k][2], clean[k][2])
+
+
+@pytest.mark.parametrize("width,height,n", [(8, 8, 40), (33, 7, 300), (61, 45, 900), (16, 16, 3000)])
+def test_marks_of_the_render(width, height, n):
+    """The render marks what blends into each block, and the backward gives the oracle's gradients from the marks."""
+    m2, d, r, c, col, op = random_scene(n, n, width, height)
+    bg = torch.tensor([0.2, 0.6, 0.4], device=DEV)
+    g = torch.Generator().manual_seed(3)
+    feats = torch.randn(n, 32, generator=g).to(DEV)
+    gi, gf = torch.randn(height, width, 3, generator=g).to(DEV), torch.randn(height, width, 32, generator=g).to(DEV)
+    ext = _get_rasterizer()
+    values, ranges, conic4, color4 = ext.bin(m2, d, r, c, col, op, width, height)
+    plain = ext.render(m2, conic4, color4, values, ranges, width, height, bg, feats)
+    marks = torch.full((4 * values.numel(),), 7, device=DEV, dtype=torch.uint8)
+    image, fimg, T, nc = ext.render(m2, conic4, color4, values, ranges, width, height, bg, feats, contributes=marks)
+    for a, b in zip(plain, (image, fimg, T, nc)):
+        assert torch.equal(a, b)
+    marked, lists, tiles, last = np_(marks), np_(values), np_(ranges), np_(nc)
+    mean, con, opac = (np_(t).astype(np.float64) for t in (m2, c, op))
+    tiles_x = (width + 15) // 16
+    for t, (begin, end) in enumerate(tiles):
+        gids = lists[begin:end]
+        for b in range(4):
+            x0, y0 = t % tiles_x * 16 + b % 2 * 8, t // tiles_x * 16 + b // 2 * 8
+            if x0 >= width or y0 >= height:
+                continue
+            ys, xs = np.mgrid[y0:min(y0 + 8, height), x0:min(x0 + 8, width)]
+            dx, dy = xs.ravel() + 0.5 - mean[gids, :1], ys.ravel() + 0.5 - mean[gids, 1:]
+            alpha = opac[gids] * np.exp(-0.5 * (con[gids, :1] * dx * dx + 2 * con[gids, 1:2] * dx * dy + con[gids, 2:] * dy * dy))
+            walked = np.arange(len(gids))[:, None] < last[y0:y0 + 8, x0:x0 + 8].ravel()
+            # Away from 1/255 by more than the rounding of alpha (a few ulp of the exponent's argument).
+            sure = (walked & (alpha > 1.0001 / 255)).any(1)
+            never = ~(walked & (alpha > 0.9999 / 255)).any(1)
+            deepest = int(last[y0:y0 + 8, x0:x0 + 8].max())
+            got = marked[4 * begin + b * len(gids):][:deepest]
+            assert (got <= 1).all() and (got[sure[:deepest]] == 1).all() and (got[never[:deepest]] == 0).all()
+    got = ext.render_backward(m2, conic4, color4, values, ranges, T, nc, width, height, grad_image=gi, background=bg,
+                              features=feats, grad_feature_image=gf, contributes=marks)
+    want = oracle.render_backward(width, height, tiles, lists, *[np_(t) for t in (m2, c, op, col)], np_(bg), np_(T), last,
+                                  np_(gi), np_(feats), np_(gf))
+    compare([np_(t) for t in got], want)
