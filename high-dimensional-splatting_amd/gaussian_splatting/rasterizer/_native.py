@@ -11,6 +11,7 @@ There is no CPU path: a missing library or a tensor off the GPU raises RuntimeEr
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 import os
@@ -147,11 +148,21 @@ class KernelProfile:
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    """The current torch stream's handle, without a Stream object made for each call."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+_CURRENT = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """Makes `device` current for a library call: nothing to do where it already is. (With plain handles for streams and
+    pointers: projection forward and backward of 1.18M gaussians, whose kernels take 51 us, 155 -> 140 us a call.)"""
+    return _CURRENT if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 _BLACK: dict[int, torch.Tensor] = {}
@@ -310,7 +321,7 @@ class HipRasterizer:
         depths = torch.empty((n,), device=means.device, dtype=torch.float32)
         radii = torch.empty((n,), device=means.device, dtype=torch.float32)
         conics = torch.empty((n, 3), device=means.device, dtype=torch.float32)
-        with torch.cuda.device(means.device):
+        with _on(means.device):
             self._run("project_forward", lambda: self.lib.hds_project_gaussians(
                 n, _ptr(means), _ptr(scales), _ptr(quats), _ptr(opacities), _ptr(pose), float(fx), float(fy),
                 float(cx), float(cy), int(width), int(height), float(near_plane), float(low_pass), float(fov_scale),
@@ -324,7 +335,7 @@ class HipRasterizer:
         means, scales, quats = _dev(means, "means"), _dev(scales, "scales"), _dev(quats, "quats")
         pose = _dev(world_to_camera, "world_to_camera")
         dm, ds, dq = torch.empty_like(means), torch.empty_like(scales), torch.empty_like(quats)
-        with torch.cuda.device(means.device):
+        with _on(means.device):
             self._run("project_backward", lambda: self.lib.hds_project_gaussians_backward(
                 means.shape[0], _ptr(gm), _ptr(gc), _ptr(means), _ptr(scales), _ptr(quats), _ptr(pose), float(fx),
                 float(fy), float(cx), float(cy), int(width), int(height), float(near_plane), float(low_pass),
@@ -339,7 +350,7 @@ class HipRasterizer:
         dirs, radii = _dev(dirs, "dirs"), _dev(radii, "radii")
         n = sh_dc.shape[0]
         rgb = torch.empty((n, 3), device=sh_dc.device, dtype=torch.float32)
-        with torch.cuda.device(sh_dc.device):
+        with _on(sh_dc.device):
             self._run("eval_sh", lambda: self.lib.hds_eval_sh(n, int(degree), _ptr(sh_dc), _ptr(sh_rest), _ptr(dirs), _ptr(radii),
                                         _ptr(rgb), _stream(sh_dc.device)))
         return rgb
@@ -353,7 +364,7 @@ class HipRasterizer:
                 raise RuntimeError(f"{name} must be a contiguous float32 CUDA tensor (updated in place)")
         grad_rgb, dirs, radii = _dev(grad_rgb, "grad_rgb"), _dev(dirs, "dirs"), _dev(radii, "radii")
         grad_dirs = torch.empty_like(dirs)
-        with torch.cuda.device(sh_dc.device):
+        with _on(sh_dc.device):
             self._run("eval_sh_backward_adam", lambda: self.lib.hds_eval_sh_backward_adam(
                 sh_dc.shape[0], int(degree), _ptr(grad_rgb), _ptr(sh_dc), _ptr(sh_rest), _ptr(dirs), _ptr(radii),
                 _ptr(m_dc), _ptr(v_dc), _ptr(m_rest), _ptr(v_rest), _ptr(step_dc), _ptr(step_rest), float(lr_dc),
@@ -377,7 +388,7 @@ class HipRasterizer:
         conic4 = torch.empty((n, 4), device=dev, dtype=torch.float32)
         color_opacity4 = torch.empty((n, 4), device=dev, dtype=torch.float32)
         tile_ranges = torch.empty((tiles, 2), device=dev, dtype=torch.int32)
-        with torch.cuda.device(dev):
+        with _on(dev):
             stream = _stream(dev)
             ws = torch.empty(self.lib.hds_bin_workspace_bytes(n, width, height), device=dev, dtype=torch.uint8)
             pairs = ctypes.c_int64(0)
@@ -430,7 +441,7 @@ class HipRasterizer:
         conic4 = torch.empty((n, 4), device=dev, dtype=torch.float32)
         color_opacity4 = torch.empty((n, 4), device=dev, dtype=torch.float32)
         tile_ranges = torch.empty((tiles, 2), device=dev, dtype=torch.int32)
-        with torch.cuda.device(dev):
+        with _on(dev):
             stream = _stream(dev)
             ws = torch.empty(self.lib.hds_bin_workspace_bytes(n, width, height), device=dev, dtype=torch.uint8)
             values = torch.empty((cap,), device=dev, dtype=torch.int32)
@@ -490,7 +501,7 @@ class HipRasterizer:
             pending.values = pending.values[:total]
             return False
         values = torch.empty((total,), device=dev, dtype=torch.int32)
-        with torch.cuda.device(dev):
+        with _on(dev):
             pws = torch.empty(self.lib.hds_pairs_workspace_bytes(total, width, height), device=dev,
                               dtype=torch.uint8)
             if not overflow:
@@ -570,7 +581,7 @@ class HipRasterizer:
                                             and contributes.dtype == torch.uint8
                                             and contributes.numel() >= 4 * values_sorted.numel()):
             raise RuntimeError("contributes must hold four uint8 per pair on the render's device")
-        with torch.cuda.device(dev):
+        with _on(dev):
             if contributes is not None:
                 self._run("render", lambda: self.lib.hds_render_contributes(
                     *args, _ptr(clear), 0 if clear is None else clear.numel(), _ptr(contributes), _stream(dev)))
@@ -623,7 +634,7 @@ class HipRasterizer:
                 values_sorted.numel(), _ptr(_dev(means2D, "means2D")), _ptr(conic4), _ptr(color_opacity4),
                 _ptr(background), _ptr(final_T), _ptr(n_contrib), _ptr(grad_image), _ptr(features),
                 _ptr(grad_feature_image), _ptr(g_means), _ptr(g_conics), _ptr(g_colors), _ptr(g_opac), _ptr(g_feat))
-        with torch.cuda.device(dev):
+        with _on(dev):
             rows, workspace = self._backward_workspace(n, int(width), int(height), channels, slice_width or 0, want_feat,
                                                        values_sorted.numel(), dev)
             if workspace is not None:
@@ -696,7 +707,7 @@ class HipRasterizer:
         n = radii.shape[0]
         if grad_means2D.shape != (n, 2) or max_radii2D.numel() != n or grad_accum.numel() != n or denom.numel() != n:
             raise RuntimeError("densification statistics need means2D_grad [N,2], radii [N] and [N] / [N,1] buffers")
-        with torch.cuda.device(radii.device):
+        with _on(radii.device):
             self._run("densification_stats", lambda: self.lib.hds_densification_stats(
                 n, _ptr(grad_means2D), _ptr(radii), int(width), int(height), _ptr(max_radii2D), _ptr(grad_accum),
                 _ptr(denom), _stream(radii.device)))
@@ -710,7 +721,7 @@ class HipRasterizer:
             raise RuntimeError("ssim inputs must both be [H, W, 3]")
         h, w = rendered.shape[0], rendered.shape[1]
         outs = [torch.empty_like(rendered) for _ in range(4)]
-        with torch.cuda.device(rendered.device):
+        with _on(rendered.device):
             self._run("ssim_forward", lambda: self.lib.hds_ssim_forward(h, w, _ptr(rendered), _ptr(gt), *[_ptr(o) for o in outs],
                                              _stream(rendered.device)))
         return tuple(outs)
@@ -721,7 +732,7 @@ class HipRasterizer:
         grad_mean = _dev(grad_mean.reshape(1).to(torch.float32), "grad_mean")
         grad = torch.empty_like(rendered)
         h, w = rendered.shape[0], rendered.shape[1]
-        with torch.cuda.device(rendered.device):
+        with _on(rendered.device):
             self._run("ssim_backward", lambda: self.lib.hds_ssim_backward(h, w, _ptr(grad_mean), _ptr(rendered), _ptr(gt), _ptr(_dev(d_mu, "d_mu")),
                                               _ptr(_dev(d_aa, "d_aa")), _ptr(_dev(d_ab, "d_ab")), _ptr(grad),
                                               _stream(rendered.device)))
