@@ -36,7 +36,7 @@
 // stores plus 0.17 ms as loads.
 //
 // Measured at 1.18M gaussians, 979x546, against the two kernels of hds_render_backward (lane = pixel, a
-// serial chain per gaussian, atomics; side by side): C = 128 lists 0.08 + replay 0.74 + sums 0.42 ms for 1.68,
+// serial chain per gaussian, atomics; side by side): C = 128 lists 0.08 + replay 0.71 + sums 0.39 ms for 1.68,
 // RGB alone 0.08 + 0.32 + 0.06 for 0.66, C = 512 4.5 for 6.4; 4M gaussians at 1920x1080, C = 256: 2.6 for 4.2. The
 // replay issues 1,290 VALU instructions per group (0.36 ms), 106 MFMAs (0.11 ms), and moves 1.3 GB of feature
 // rows in and 1.5 GB of gradient rows out; it runs two waves per SIMD (250 VGPRs, 40 KB of LDS per block).
@@ -731,8 +731,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
 					for (int u = 0; u < 2; u++) {
 						float* p = to + (S / 4) * u;
+						// Whole lines, read again only after the launch: past the caches, which keep the feature rows
+						// (1.18M, C = 128: replay 0.734 -> 0.708 ms, sums 0.414 -> 0.393; non-temporal reads of the rows save
+						// 0.010 more there and cost 0.003 of 0.037 at 200k, C = 32).
 						if constexpr (kKc == 4)
-							*reinterpret_cast<float4*>(p) = make_float4(D[u][0][i], D[u][1][i], D[u][2][i], D[u][3][i]);
+							__builtin_nontemporal_store(hds_f32x4{D[u][0][i], D[u][1][i], D[u][2][i], D[u][3][i]}, reinterpret_cast<hds_f32x4*>(p));
 						else if constexpr (kKc == 2)
 							*reinterpret_cast<float2*>(p) = make_float2(D[u][0][i], D[u][1][i]);
 						else

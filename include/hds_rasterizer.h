@@ -228,8 +228,8 @@ HDS_API int hds_render(int64_t n, int width, int height, int channels, const int
 			   float* feature_image, hds_stream_t stream);
 
 /* hds_render that also zeroes `clear_count` floats at `clear` (16-byte aligned, a multiple of 4;
- * 0 clears nothing), each tile's work-group one share before its walk: the zero-initialised
- * gradient buffers of a following hds_render_backward_accumulate, cleared in the bandwidth the
+ * 0 clears nothing), each work-group a share before its walk: the zero-initialised gradient buffers of a
+ * following hds_render_backward_rows or hds_render_backward_accumulate, cleared in the bandwidth the
  * walk leaves unused instead of by a fill of their own. The same results as hds_render followed by
  * hds_zero_async over the range; the range must not overlap the render's inputs or outputs. No
  * counterpart in the reference, which allocates its gradient
@@ -325,8 +325,8 @@ HDS_API int hds_densification_stats(int64_t n, const float* grad_means2D, const 
 
 /* ---- kernel timing (no counterpart in the reference; for benchmarks) ------------------------ */
 
-/* Starts recording: from now on every hot-path kernel launch (projection, blend forward, the two
- * blend-backward kernels) is bracketed by HIP events on its own stream. Clears earlier records. */
+/* Starts recording: from now on every hot-path kernel launch (projection, binning, blend forward and
+ * backward, SH, SSIM) is bracketed by HIP events on its own stream. Clears earlier records. */
 HDS_API int hds_profile_begin(void);
 
 /* hds_profile_begin restricted to the kernels named in `kernels`, a comma-separated list of kernel
