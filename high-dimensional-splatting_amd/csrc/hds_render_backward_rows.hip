@@ -37,7 +37,7 @@
 //
 // Measured at 1.18M gaussians, 979x546, against the two kernels of hds_render_backward (lane = pixel, a
 // serial chain per gaussian, atomics; side by side): C = 128 lists 0.08 + replay 0.71 + sums 0.39 ms for 1.68,
-// RGB alone 0.08 + 0.32 + 0.06 for 0.66, C = 512 4.5 for 6.4; 4M gaussians at 1920x1080, C = 256: 2.6 for 4.2. The
+// RGB alone 0.08 + 0.27 + 0.06 for 0.66, C = 512 4.5 for 6.4; 4M gaussians at 1920x1080, C = 256: 2.6 for 4.2. The
 // replay issues 1,290 VALU instructions per group (0.36 ms), 106 MFMAs (0.11 ms), and moves 1.3 GB of feature
 // rows in and 1.5 GB of gradient rows out; it runs two waves per SIMD (250 VGPRs, 40 KB of LDS per block).
 #include <algorithm>
@@ -340,8 +340,10 @@ __device__ inline float fold16(float a, float b) {
 
 // REST: the second launch where the rows might not fit: it returns at once when they did, and otherwise adds the
 // gradients of the rows past the capacity atomically.
+// RGB alone fits three waves per SIMD (167 VGPRs; 0.317 -> 0.270 ms at 1.18M gaussians, 979x546); a slice of 32 channels
+// would spill 16 registers for it and gains nothing.
 template <int S, bool RGB, bool WANT, bool REST>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void backward_geometry_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(S == 0 ? 3 : 2))) void backward_geometry_kernel(
 	const BackwardArgs a) {
 	constexpr int kKc = S > 0 ? S / 32 : 1;    // K steps of the dot products
 	constexpr int kRun = S > 0 ? S / 8 : 4;    // channels per run of an F row
